@@ -17,7 +17,7 @@ struct GView {
     float orient;        // sign of cross(b, a): cross(b, X - S) * orient > 0 in front
     int32_t t0;          // rows (z order) whose ray does not rise (dz <= 0); set by the gather pre-pass
     float szlo;          // sz's FP32 rounding residual: the source height is sz + szlo
-    float pad[2];
+    double kb;           // -dz0 / dzs + 1/2 in FP64: tau + 1/2 of the plane through the source
 };
 static_assert(sizeof(GView) == 64, "GView layout");
 
@@ -61,6 +61,7 @@ __device__ inline bool gather_view(const RayCfg& rc, const ap_proj_spec* __restr
     gv.szlo = (float)(Sz - (double)gv.sz);
     gv.dz0 = (float)(vr.Q00[2] + kv_first * vz - vr.S[2]);
     gv.dzs = (float)(fabs(vz) / ssv);
+    gv.kb = 0.5 - (vr.Q00[2] + kv_first * vz - vr.S[2]) / (fabs(vz) / ssv);
     gv.sx = (float)Sx;
     gv.sy = (float)Sy;
     gv.ax = (float)ax;
@@ -74,11 +75,13 @@ __device__ inline bool gather_view(const RayCfg& rc, const ap_proj_spec* __restr
 
 
 // Bytes of workspace the gather adjoint needs for V views (0 for an empty
-// problem); whether it supports nv x ssv sub-rows; and its launch (returns
+// problem) and the bytes behind them that it can use for partial sums; whether
+// it supports nv x ssv sub-rows; and its launch (returns
 // AP_ERR_UNSUPPORTED when it cannot take the call).  With `left`, the launch
 // also counts the views it does not take into the workspace and returns that
 // device counter there.
 uint64_t gather_workspace_bytes(uint32_t V, uint32_t nu, uint32_t nv, uint32_t ssu, uint32_t ssv);
+uint64_t gather_partial_bytes(uint32_t V, uint64_t tables);
 bool gather_supported(uint32_t nv, uint32_t ssv);
 int32_t launch_gather_adjoint(const RayCfg& rc, uint32_t V, uint32_t nu, uint32_t nv, int64_t s0, int64_t s1,
                               int64_t s2, uint32_t ssu, uint32_t ssv, double scale, const ap_proj_spec* specs,

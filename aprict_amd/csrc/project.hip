@@ -600,5 +600,7 @@ extern "C" uint64_t ap_backproject_matched_workspace_size(const ap_config_cb_pro
                                                           const ap_array3* sino_desc) {
     if (!cfg || !sino_desc || cfg->ssu < 1 || cfg->ssv < 1) return 0;
     if (!gather_supported(sino_desc->shape[2], cfg->ssv)) return 0;
-    return gather_workspace_bytes(num_projs, sino_desc->shape[1], sino_desc->shape[2], cfg->ssu, cfg->ssv);
+    const uint64_t tables =
+        gather_workspace_bytes(num_projs, sino_desc->shape[1], sino_desc->shape[2], cfg->ssu, cfg->ssv);
+    return tables + gather_partial_bytes(num_projs, tables);
 }

@@ -28,15 +28,17 @@ constexpr int kGbcRows = 2;   // voxel rows per workgroup of the GBC kernel
 //   the detector centre, geometry.py:75-107 expanded into a projective map),
 //   lambda = K/(W.x + w0) is the source->detector / source->point ratio,
 //   Z = Zc.x + z0 is the distance along the source->detector-centre axis.
-struct ViewMap {
-    float Au[3], au, Av[3], av, W[3], w0, K;
-    float Zc[3], z0, Lnorm;
-    float S[3], D[3], U[3], Vv[3];
-    float nu, nv, uvnorm;
-    float kq;              // K^2 / (|u| |v|): the FDK weight is kq w^3 / (W.x + w0)^2
+// In groups of four, so that a wave reads each group from LDS at once.
+struct alignas(16) ViewMap {
+    float Au[3], au, Av[3], av, W[3], w0, Zc[3], z0;
     float hu, hv;          // (nu - 1) / 2, (nv - 1) / 2: pixel index of the detector centre
+    float kq;              // K^2 / (|u| |v|): the FDK weight is kq w^3 / (W.x + w0)^2
+    float inv_Lnorm;       // 1 / |D - S|
     float inv_hnu, inv_hnv;   // 2 / nu, 2 / nv
-    float inv_Lnorm;          // 1 / |D - S|
+    float K, Lnorm;
+    float S[3], inv_Sxy;      // source, 1 / its distance from the z axis
+    float D[3], U[3], Vv[3];
+    float nu, nv, uvnorm;
 };
 
 __device__ void make_view_map(const ap_proj_spec* specs, uint32_t p, ViewMap& m) {
@@ -121,6 +123,7 @@ struct BpCfg {
     float inv_sep;        // 1 / sep (0 when sep == 0)
     float w3;             // voxwid^3
     bool off32;           // detector offsets of one view fit 32 bits
+    bool bytes32;         // its byte offsets too, and FP32 holds the edge tests' bounds (sides below 2^22)
     bool pair;            // v contiguous (s2 == 1), nv >= 2, 32-bit offsets: rows k, k+1 in one load
     bool grouped;         // bp_col_views over 4 views applies: offsets of 4 views fit 32 bits (and pairs if bilinear)
     int zl, zv;
@@ -509,6 +512,157 @@ __device__ __forceinline__ void bp_col_views(const BpCfg& c, const ViewMap* Ms, 
             acc[m] += mult[v][m] == 0.f ? 0.f : soften(c, Ms[v], cu[v][m], cv[v][m], y[v][m] * mult[v][m]);
 }
 
+// u part of a z-coherent view at (x0, x1): what a voxel column shares.
+struct ColView {
+    float cu, cv0, dcv;   // cu; cv = fma(z, dcv, cv0)
+};
+__device__ __forceinline__ ColView col_view(const ViewMap& M, float x0, float x1, float& iw) {
+    const float wx = M.W[0] * x0 + M.W[1] * x1 + M.w0;
+    iw = __builtin_amdgcn_rcpf(wx);
+    return ColView{(M.Au[0] * x0 + M.Au[1] * x1 + M.au) * iw, (M.Av[0] * x0 + M.Av[1] * x1 + M.av) * iw,
+                   M.Av[2] * iw};
+}
+
+// Detector reads of a z-coherent view at kZ voxels of a column whose taps all
+// lie on the detector: no clamps, no range flags.  cv grows or falls with z
+// throughout, so the caller's test of the first and last voxel covers those
+// between.  The values are those of sample_det.
+// Addresses are the view's scalar base plus one 32-bit byte offset per voxel;
+// the second tap column has a scalar base of its own.  The two rows of a tap
+// column come in one load: a wave's gather of 8-byte pairs takes the L1 as long
+// as two of 4 bytes (18 and 9 cycles), in half the instructions (four separate
+// loads: 6.9 against 5.0 ms for the FDK backprojection at 256^3 x 360 x 384^2).
+template <int kZ, typename Tp>
+struct ColTaps {
+    TapPair<Tp> pa[kZ], pb[kZ];
+    float ta, tb[kZ];
+    Tp yn[kZ];   // nearest
+};
+template <typename T>
+__device__ __forceinline__ T at_byte(const void* base, uint32_t o) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + o);
+}
+template <int kZ, typename Tp>
+__device__ __forceinline__ void col_taps(const BpCfg& c, const ViewMap& M, const ColView& V,
+                                         const Tp* __restrict__ img, const float (&z)[kZ], ColTaps<kZ, Tp>& t) {
+    const float fj = V.cu + M.hu;
+    const uint32_t es = (uint32_t)sizeof(Tp);
+    if (c.bilinear) {
+        const float flj = floorf(fj);
+        t.ta = fj - flj;
+        const uint32_t oj = (uint32_t)(int)flj * ((uint32_t)c.s1 * es);
+        const Tp* img1 = img + c.s1;
+#pragma unroll
+        for (int m = 0; m < kZ; m++) {
+            const float fk = __builtin_fmaf(z[m], V.dcv, V.cv0) + M.hv;
+            const float flk = floorf(fk);
+            t.tb[m] = fk - flk;
+            const uint32_t o = (uint32_t)(int)flk * es + oj;
+            t.pa[m] = at_byte<TapPair<Tp>>(img, o);
+            t.pb[m] = at_byte<TapPair<Tp>>(img1, o);
+        }
+    } else {
+        const uint32_t oj = (uint32_t)(int)floorf(fj + 0.5f) * ((uint32_t)c.s1 * es), ek = (uint32_t)c.s2 * es;
+#pragma unroll
+        for (int m = 0; m < kZ; m++) {
+            const float fk = __builtin_fmaf(z[m], V.dcv, V.cv0) + M.hv;
+            t.yn[m] = at_byte<Tp>(img, (uint32_t)(int)floorf(fk + 0.5f) * ek + oj);
+        }
+    }
+}
+template <int kZ, typename Tp>
+__device__ __forceinline__ float col_value(const BpCfg& c, const ColTaps<kZ, Tp>& t, int m) {
+    if (!c.bilinear) return to_f32(t.yn[m]);
+    const float a = t.ta, b = t.tb[m];
+    const float t1 = to_f32(t.pa[m].lo) * (1.f - a) + to_f32(t.pb[m].lo) * a;
+    const float t2 = to_f32(t.pa[m].hi) * (1.f - a) + to_f32(t.pb[m].hi) * a;
+    return t1 * (1.f - b) + t2 * b;
+}
+// Whether every tap of the column's voxels from zf to zl is on the detector.
+__device__ __forceinline__ bool col_inside(const BpCfg& c, const ViewMap& M, const ColView& V, float zf, float zl) {
+    const float fj = V.cu + M.hu;
+    const float f0 = __builtin_fmaf(zf, V.dcv, V.cv0) + M.hv, f1 = __builtin_fmaf(zl, V.dcv, V.cv0) + M.hv;
+    const float lo = fminf(f0, f1), hi = fmaxf(f0, f1);
+    if (!c.bytes32) return false;
+    if (c.bilinear) return fj >= 0.f && lo >= 0.f && fj < (float)(c.nu - 1) && hi < (float)(c.nv - 1);
+    return fj > -0.5f && lo > -0.5f && fj < (float)c.nu - 0.75f && hi < (float)c.nv - 0.75f;
+}
+
+// kV consecutive z-coherent views at kZ voxels of one column.  Where every tap
+// of the wave's active voxels is on the detector and outside the softening
+// band -- one test per column and view, of the first and last voxel -- a voxel
+// costs the interpolation alone; elsewhere bp_col_views takes the views, with
+// the same sums.  Clamps, range flags, the softening test and 64-bit addresses
+// were two thirds of a voxel's instructions; what is left is bound about
+// equally by the vector units (35 instructions a voxel and view) and the L1's
+// gathers (36 cycles).  FDK at 256^3 from 360 views of 384^2, ramp filter
+// included: 7.8 -> 5.5 ms; nearest pixels at 256^3 from 180 views of 512^2
+// (a SIRT step's backprojection): 6.6 -> 3.1 ms.
+template <int kV, int kZ, typename Tp>
+__device__ __forceinline__ void bp_coherent(const BpCfg& c, const ViewMap* Ms, const Tp* __restrict__ img,
+                                            int64_t s0, float x0, float x1, const float (&z)[kZ], float zl,
+                                            uint32_t act, float (&acc)[kZ]) {
+    ColView V[kV];
+    float mult[kV];
+    bool inside = true;
+#pragma unroll
+    for (int v = 0; v < kV; v++) {
+        const ViewMap& M = Ms[v];
+        float iw;
+        V[v] = col_view(M, x0, x1, iw);
+        float mu = c.direct ? 1.f : M.kq * c.w3 * (iw * iw);
+        const bool pre = c.direct && c.preset != 0;
+        if (c.zl != 0 || c.zv != 0 || pre) {
+            const float zz = M.Zc[0] * x0 + M.Zc[1] * x1 + M.z0;
+            if (c.zl != 0) mu *= powi(zz * M.inv_Lnorm, c.zl);
+            if (c.zv != 0) mu *= powi(zz * c.inv_zval, c.zv);
+            if (pre) {
+                const float xp[3] = {x0, x1, 0.f};   // the presets use x and y only
+                mu = apply_preset(c, M, xp, zz, mu);
+            }
+        }
+        mult[v] = mu;
+        inside = inside && mu != 0.f && col_inside(c, M, V[v], z[0], zl);
+        if (c.sep > 0.f) {
+            // no voxel in the softening band: both ramps at 1 at both ends
+            const float ud = (1.f - fabsf(V[v].cu) * M.inv_hnu) * c.inv_sep;
+            const float va = fmaxf(fabsf(__builtin_fmaf(z[0], V[v].dcv, V[v].cv0)),
+                                   fabsf(__builtin_fmaf(zl, V[v].dcv, V[v].cv0)));
+            inside = inside && ud >= 1.f && (1.f - va * M.inv_hnv) * c.inv_sep >= 1.f;
+        }
+    }
+    if (__ballot(!inside) != 0) {
+        if constexpr (kV == 1) {
+            bp_col_views<1, kZ, true>(c, Ms, img, s0, x0, x1, z, act, acc);
+        } else {
+            // one voxel and view at a time: a group's registers would be the kernel's
+#pragma unroll
+            for (int v = 0; v < kV; v++)
+#pragma unroll
+                for (int m = 0; m < kZ; m++) {
+                    const float zm[1] = {z[m]};
+                    float am[1] = {acc[m]};
+                    bp_col_views<1, 1, true>(c, Ms + v, img + v * (int32_t)s0, s0, x0, x1, zm, (act >> m) & 1u, am);
+                    acc[m] = am[0];
+                }
+        }
+        return;
+    }
+    ColTaps<kZ, Tp> t[kV];
+#pragma unroll
+    for (int v = 0; v < kV; v++) col_taps<kZ>(c, Ms[v], V[v], img + v * (int32_t)s0, z, t[v]);
+    {
+#pragma clang fp contract(off)   // the sums of bp_col_views, which adds a rounded product
+#pragma unroll
+        for (int v = 0; v < kV; v++)
+#pragma unroll
+            for (int m = 0; m < kZ; m++) {
+                const float val = col_value<kZ>(c, t[v], m) * mult[v];
+                acc[m] += val;
+            }
+    }
+}
+
 template <typename Tp>
 __device__ float bp_one_view(const BpCfg& c, const ViewMap& m, const Tp* __restrict__ img,
                              const float x[3]) {
@@ -561,19 +715,30 @@ __device__ float bp_one_view(const BpCfg& c, const ViewMap& m, const Tp* __restr
 }
 
 // One thread per kZ voxels of a column, kBz apart along z (a wave holds kBz
-// consecutive voxels at each of its kZ heights).  The interpolating branch
-// without sub-voxel sampling runs bp_col_views, with the shared u part on a
-// batch of views that are all z-coherent; the host takes kZ > 1 only there.
-// A voxel's sum is the same for every kZ and launch shape.
-template <int kBy, int kZ, typename Tv, typename Tp, typename Tm>
-__global__ __launch_bounds__(kBz* kBy) void k_backproject_voxel(
+// consecutive voxels at each of its kZ heights).  kCols: the interpolating
+// branch without sub-voxel sampling, bp_coherent on a batch of views that are
+// all z-coherent, else bp_col_views.  Otherwise (kZ = 1) the exact branch,
+// sub-voxel sampling, unpaired taps and 64-bit detector offsets, apart so that
+// their registers are not the columns'.
+// A voxel's sum is the same for every kZ and launch shape.  7 waves per SIMD
+// for tall columns: with 5, 6 and 8 the nearest-pixel case of bp_coherent takes
+// 8.1, 7.6 and 8.8 ms a SIRT step against 7.0 (at 8 it spills in the view loop),
+// the bilinear one the same from 5 to 7.  5 where a thread takes four (view,
+// voxel) pairs from two views or more (kZ <= 2): they hold four views' maps, and
+// 7 waves spill them.
+// Nearest pixels of kZ <= 2 stay with bp_col_views: a clamp and a flag per voxel
+// cost less there than the column's test, which waits for a ballot before the
+// first load (62 planes and fewer, 40 to 390 views: 0.97 against 1.2 to 1.45 of
+// the time of the general path).
+template <bool kCols, int kZ, typename Tv, typename Tp, typename Tm>
+__global__ __launch_bounds__(kBz* kBpRowsY[0], kCols ? (kZ <= 2 ? 5 : 7) : 4) void k_backproject_voxel(
     BpCfg c, const ap_proj_spec* __restrict__ specs, uint32_t num_projs,
     Tv* __restrict__ vol, int64_t vs0, int64_t vs1, int64_t vs2,
     const Tm* __restrict__ mult, int64_t ms0, int64_t ms1, int64_t ms2,
     const Tp* __restrict__ sino) {
     __shared__ ViewMap maps[kViewBatch];
     const uint32_t ck0 = blockIdx.x * (kBz * kZ) + threadIdx.x;
-    const uint32_t cj = blockIdx.y * kBy + threadIdx.y;
+    const uint32_t cj = blockIdx.y * blockDim.y + threadIdx.y;
     const uint32_t ci = blockIdx.z;
     const uint32_t gi = ci + c.off[0], gj = cj + c.off[1];
     const float x0 = c.c000[0] + (float)gi * c.w, x1 = c.c000[1] + (float)gj * c.w;
@@ -588,12 +753,13 @@ __global__ __launch_bounds__(kBz* kBy) void k_backproject_voxel(
         const uint32_t ck = ck0 + (uint32_t)(kBz * m);
         z[m] = c.c000[2] + (float)(ck + c.off[2]) * c.w;
         if (col_in && ck < c.shp[2]) act |= 1u << m;
+        else if (m > 0) z[m] = z[m - 1];   // past the column: reads where its last voxel reads
         acc[m] = 0.f;
     }
+    const float zl = z[kZ - 1];
     asm volatile("" : "+v"(act));
     const bool any = act != 0;
     const uint32_t nss = c.ssx * c.ssy * c.ssz;
-    const bool zcol = !c.exact && nss == 1 && (c.bilinear ? c.pair : c.off32);
     const int tid = threadIdx.y * kBz + threadIdx.x;
     for (uint32_t p0 = 0; p0 < num_projs; p0 += kViewBatch) {
         const uint32_t nb = min((uint32_t)kViewBatch, num_projs - p0);
@@ -606,30 +772,31 @@ __global__ __launch_bounds__(kBz* kBy) void k_backproject_voxel(
         // every view of the batch z-coherent (the barrier publishes the maps)
         const bool batch_z = __syncthreads_and(coherent) != 0;
         if (!any || nss != 1) continue;
-        if (zcol) {
+        if constexpr (kCols) {
             const Tp* img = sino + (int64_t)p0 * c.s0;
             uint32_t q = 0;
-            if constexpr (kZ == 1) {
+            // four (view, voxel) pairs at a time
+            constexpr int kV = kZ == 1 ? 4 : kZ == 2 ? 2 : 1;
+            if constexpr (kV > 1) {
                 if (c.grouped) {
-                    for (; q + 4 <= nb; q += 4) {
-                        if (batch_z)
-                            bp_col_views<4, 1, true>(c, maps + q, img + (int64_t)q * c.s0, c.s0, x0, x1, z, act, acc);
+                    for (; q + kV <= nb; q += kV) {
+                        const Tp* im = img + (int64_t)q * c.s0;
+                        if (batch_z && c.bilinear)
+                            bp_coherent<kV, kZ>(c, maps + q, im, c.s0, x0, x1, z, zl, act, acc);
+                        else if (batch_z)
+                            bp_col_views<kV, kZ, true>(c, maps + q, im, c.s0, x0, x1, z, act, acc);
                         else
-                            bp_col_views<4, 1, false>(c, maps + q, img + (int64_t)q * c.s0, c.s0, x0, x1, z, act, acc);
+                            bp_col_views<kV, kZ, false>(c, maps + q, im, c.s0, x0, x1, z, act, acc);
                     }
                 }
             }
             for (; q < nb; q++) {
                 if (batch_z)
-                    bp_col_views<1, kZ, true>(c, maps + q, img + (int64_t)q * c.s0, c.s0, x0, x1, z, act, acc);
+                    bp_coherent<1, kZ>(c, maps + q, img + (int64_t)q * c.s0, c.s0, x0, x1, z, zl, act, acc);
                 else
                     bp_col_views<1, kZ, false>(c, maps + q, img + (int64_t)q * c.s0, c.s0, x0, x1, z, act, acc);
             }
-            continue;
-        }
-        if constexpr (kZ == 1) {
-            // the exact branch, and the interpolating branch with unpaired taps or
-            // 64-bit detector offsets, voxel by voxel
+        } else {
             const float xc[3] = {x0, x1, z[0]};
             if (c.exact) {
                 for (uint32_t q = 0; q < nb; q++)
@@ -640,12 +807,10 @@ __global__ __launch_bounds__(kBz* kBy) void k_backproject_voxel(
             }
         }
     }
-    if (nss != 1) {
-        // general sub-voxel sampling (kZ = 1 only): views re-derived per sub-voxel
-        // (CB_backproject.cu:377-383 loop order: x, y, z outermost to innermost)
-#pragma unroll
-        for (int m = 0; m < kZ; m++) {
-            if (!((act >> m) & 1u)) continue;
+    if constexpr (!kCols) {
+        if (nss != 1 && any) {
+            // general sub-voxel sampling: views re-derived per sub-voxel
+            // (CB_backproject.cu:377-383 loop order: x, y, z outermost to innermost)
             float ax = 0.f;
             for (uint32_t si = 0; si < c.ssx; si++) {
                 float ay = 0.f;
@@ -654,7 +819,7 @@ __global__ __launch_bounds__(kBz* kBy) void k_backproject_voxel(
                     for (uint32_t sk = 0; sk < c.ssz; sk++) {
                         const float xs[3] = {x0 + (-0.5f + (0.5f + si) / c.ssx) * c.w,
                                              x1 + (-0.5f + (0.5f + sj) / c.ssy) * c.w,
-                                             z[m] + (-0.5f + (0.5f + sk) / c.ssz) * c.w};
+                                             z[0] + (-0.5f + (0.5f + sk) / c.ssz) * c.w};
                         float a = 0.f;
                         for (uint32_t p = 0; p < num_projs; p++) {
                             ViewMap vm;
@@ -667,7 +832,7 @@ __global__ __launch_bounds__(kBz* kBy) void k_backproject_voxel(
                 }
                 ax += ay / c.ssy;
             }
-            acc[m] = ax / c.ssx;
+            acc[0] = ax / c.ssx;
         }
     }
 #pragma unroll
@@ -889,18 +1054,23 @@ int32_t launch_backproject_voxel(const ap_config_cb_backproject* cfg, const ap_p
     c.w3 = c.w * c.w * c.w;
     c.off32 = (double)(c.nu ? c.nu - 1 : 0) * (double)c.s1 + (double)(c.nv ? c.nv - 1 : 0) * (double)c.s2 <
               2147483647.0;
+    c.bytes32 = ((double)(c.nu ? c.nu - 1 : 0) * (double)c.s1 + (double)(c.nv ? c.nv - 1 : 0) * (double)c.s2 + 1.0) *
+                        dtype_size(sino_desc->dtype) < 4294967296.0 &&
+                c.nu < (1u << 22) && c.nv < (1u << 22);
     c.pair = c.off32 && c.s2 == 1 && c.nv >= 2;
     c.grouped = !c.exact && (c.bilinear ? c.pair : c.off32) &&
                 (double)c.s0 * 3.0 + (double)(c.nu ? c.nu - 1 : 0) * (double)c.s1 +
                         (double)(c.nv ? c.nv - 1 : 0) * (double)c.s2 < 2147483647.0;
     const int var = ap_tune_variant(AP_TUNE_BACKPROJECT);
     const uint32_t rows_y = (uint32_t)kBpRowsY[var];
-    // four voxels per thread along z where a column is taller than two waves'
-    // worth and the interpolating branch runs bp_col_views (which shares a
-    // z-coherent view's u part between them)
+    // Where a column is taller than a wave and the interpolating branch runs on
+    // 32-bit offsets: up to four voxels per thread along z, which share a
+    // z-coherent view's u part; as few as cover the column in ceil(nz / 256) parts.
     const uint32_t nss = c.ssx * c.ssy * c.ssz;
-    const bool z4 = !c.exact && nss == 1 && (c.bilinear ? c.pair : c.off32) && c.shp[2] > 2 * (uint32_t)kBz;
-    const uint32_t zper = z4 ? 4u * kBz : (uint32_t)kBz;
+    const bool zcol = !c.exact && nss == 1 && (c.bilinear ? c.pair : c.off32);
+    const uint32_t parts = (c.shp[2] + 4u * kBz - 1) / (4u * kBz);
+    const uint32_t kz = zcol ? (c.shp[2] + parts * kBz - 1) / (parts * kBz) : 1u;
+    const uint32_t zper = kz * kBz;
     dim3 block(kBz, rows_y, 1);
     dim3 grid((c.shp[2] + zper - 1) / zper, (c.shp[1] + rows_y - 1) / rows_y, c.shp[0]);
     const int32_t mdt = multiplier ? mult_desc->dtype : vol_desc->dtype;
@@ -930,15 +1100,11 @@ int32_t launch_backproject_voxel(const ap_config_cb_backproject* cfg, const ap_p
                                            vol_desc->strides[0], vol_desc->strides[1], vol_desc->strides[2],
                                            (const Tm*)multiplier, ms[0], ms[1], ms[2], (const Tp*)sino);
                     };
-                    if (z4) {
-                        if (var == 0) launch(k_backproject_voxel<kBpRowsY[0], 4, Tv, Tp, Tm>);
-                        if (var == 1) launch(k_backproject_voxel<kBpRowsY[1], 4, Tv, Tp, Tm>);
-                        if (var == 2) launch(k_backproject_voxel<kBpRowsY[2], 4, Tv, Tp, Tm>);
-                    } else {
-                        if (var == 0) launch(k_backproject_voxel<kBpRowsY[0], 1, Tv, Tp, Tm>);
-                        if (var == 1) launch(k_backproject_voxel<kBpRowsY[1], 1, Tv, Tp, Tm>);
-                        if (var == 2) launch(k_backproject_voxel<kBpRowsY[2], 1, Tv, Tp, Tm>);
-                    }
+                    if (!zcol) launch(k_backproject_voxel<false, 1, Tv, Tp, Tm>);
+                    else if (kz == 1) launch(k_backproject_voxel<true, 1, Tv, Tp, Tm>);
+                    else if (kz == 2) launch(k_backproject_voxel<true, 2, Tv, Tp, Tm>);
+                    else if (kz == 3) launch(k_backproject_voxel<true, 3, Tv, Tp, Tm>);
+                    else launch(k_backproject_voxel<true, 4, Tv, Tp, Tm>);
                     return ap_check_launch("backproject_voxel");
                 }
             });

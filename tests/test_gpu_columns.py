@@ -5,7 +5,7 @@ column, panels that hold every tap (no edge handling), panels that cut the
 column, and voxel columns in the softening band; v-contiguous data, a slice of
 wider data (odd strides, odd start) and fp16.  Relative L2 <= 2e-5 as for the
 other interpolating backprojections (FP32 coordinates: 2^-24 of some 50 pixels
-against pixel differences of order 1 is 3e-6 per sample).
+against pixel differences of order 1 is 3e-6 per sample), 1e-5 for GBC.
 
 Nearest-pixel reads flip where a coordinate lies within FP32 rounding of a
 pixel edge, so those cases use data that is constant along v in blocks and
@@ -82,3 +82,33 @@ def test_columns_match_oracle(device, nz, kind, name):
     assert np.abs(want).max() > 0
     # a flipped pixel moves a value by 1/40 of its neighbours' size; at most a few in 10^4 samples do
     assert err <= (5e-4 if kind == "nearest" else 2e-5)
+
+
+@pytest.mark.parametrize("name", ["f32", "slice", "f16"])
+@pytest.mark.parametrize("nz", HEIGHTS)
+@pytest.mark.parametrize("mixed", [False, True], ids=["upright", "mixed"])
+def test_gbc_columns_match_oracle(device, mixed, nz, name):
+    # the second batch of views tilted in "mixed": both routes add to one sum
+    rng = np.random.default_rng(500 + nz)
+    views, nu = (70 if mixed else 6), 31
+    shape, w = (5, 6, nz), 3.2 / 6
+    nv = max(9, int(2.3 * nz * w) | 1) if nz != 193 else 41
+    pg = panels(views, nu, nv, 0.3 * nz * w)
+    if mixed:
+        c, s = np.cos(0.05), np.sin(0.05)
+        du, dv = pg.det_uvec.copy(), pg.det_vvec.copy()
+        du[64:], dv[64:] = (c * pg.det_uvec + s * pg.det_vvec)[64:], (c * pg.det_vvec - s * pg.det_uvec)[64:]
+        pg = cbfp.ProjGeom(source_pos=pg.source_pos, det_pos=pg.det_pos, det_uvec=du, det_vvec=dv, nu=nu, nv=nv)
+    y, yy = layout(rng.uniform(-1, 2, (views, nu, nv)).astype(np.float32), name)
+    cfg = cbfp.ConfigBackproject(fast_approx=True, backproj_weighting_preset=7, Z_on_val_factor_val=40.0,
+                                 approx_mode_bilinear_interpolate=True, soft_vartheta_v=0.4,
+                                 soft_vartheta_v_softspan=0.2, soft_vartheta_h=0.06, soft_vartheta_h_softspan=0.04)
+    v = Volume(np.zeros(shape, np.float32), voxwid=w)
+    sec = Volume(np.zeros(shape, np.float32), voxwid=w)
+    cbfp.backproject(cfg, v, cbfp.ProjectionSet(pg, data=y), secondary_volume=sec, block=True)
+    wv, ws = orc.backproject_gbc(cfg.contents, pg.to_proj_spec_array(), chunk_for(shape, w), np.zeros(shape),
+                                 np.zeros(shape), yy)
+    e1, e2 = rel_l2(v.as_numpy(), wv), rel_l2(sec.as_numpy(), ws)
+    print(f"GBC columns nz={nz} {name} mixed={mixed}: values {e1:.3e}, weights {e2:.3e}")
+    assert np.abs(ws).max() > 0
+    assert e1 <= 2e-5 and e2 <= 1e-5

@@ -50,6 +50,21 @@ __device__ __forceinline__ float tcross(float pn, float r, float c) {
     return __builtin_fmaf(pn, r, c);
 }
 
+// 1 / x and 1 / sqrt(x) for a finite x away from zero: the hardware estimate and two
+// Newton steps (about 2e-16 relative; a division or square root is 10 to 20
+// instructions, of which a ray's set-up had ten)
+__device__ __forceinline__ double ray_rcp(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(fma(-x, y, 1.0), y, y);
+    return fma(fma(-x, y, 1.0), y, y);
+}
+__device__ __forceinline__ double ray_rsq(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    const double h = 0.5 * x;
+    y = fma(fma(-h * y, y, 0.5), y, y);
+    return fma(fma(-h * y, y, 0.5), y, y);
+}
+
 // FP64 -> FP32 per-view constants (CB_project_texture_chunked.cu:308-324 for
 // the pixel centres: centre of pixel (j,k) = pos + (j-(nu-1)/2) u + (k-(nv-1)/2) v).
 __device__ inline ViewRays make_view_rays(const RayCfg& rc, const ap_proj_spec* __restrict__ specs,
@@ -85,9 +100,9 @@ __device__ inline bool ray_setup(const ViewRays& vr, const int lo[3], const int 
     }
     const double l2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
     if (!(l2 > 0.0)) return false;
-    const double len = sqrt(l2);
+    const double il = ray_rsq(l2), len = l2 * il;
     double u[3];
-    for (int a = 0; a < 3; a++) u[a] = d[a] / len;
+    for (int a = 0; a < 3; a++) u[a] = d[a] * il;
     // closest approach to the chunk centre: parameter tc (distance from the source)
     const double tc = -(vr.S[0] * u[0] + vr.S[1] * u[1] + vr.S[2] * u[2]);
     float te = (float)(-tc), tx = (float)(len - tc);
@@ -109,8 +124,9 @@ __device__ inline bool ray_setup(const ViewRays& vr, const int lo[3], const int 
         const double P0 = floor(oab);
         R.P0[a] = (float)P0;
         R.sg[a] = u[a] > 0.0 ? 1 : -1;
-        R.r[a] = (float)(1.0 / u[a]);
-        R.c[a] = (float)((P0 - oab) / u[a]);
+        const double ru = ray_rcp(u[a]);
+        R.r[a] = (float)ru;
+        R.c[a] = (float)((P0 - oab) * ru);
         const float ein = (float)(R.sg[a] > 0 ? lo[a] : hi[a]) - R.P0[a];
         const float eout = (float)(R.sg[a] > 0 ? hi[a] : lo[a]) - R.P0[a];
         te = fmaxf(te, tcross(ein, R.r[a], R.c[a]));
@@ -190,19 +206,24 @@ struct Walker {
     // weight w of voxel `off`; advances state; false when this was the last voxel
     __device__ __forceinline__ bool step(float& w, IdxT& o) {
         const float tmn = fminf(fminf(tx, ty), tz);
-        const float tcl = fminf(tmn, tend);
+        const bool more = !(tmn >= tend);
+        const float tcl = more ? tmn : tend;
         w = fmaxf(tcl - tprev, 0.f);
         o = off;
         tprev = tcl;
-        if (tmn >= tend) return false;
-        if (tx == tmn) {
-            px += gx; tx = tcross(px, rx, cx); off += dox;
-        } else if (ty == tmn) {
-            py += gy; ty = tcross(py, ry, cy); off += doy;
-        } else {
-            pz += gz; tz = tcross(pz, rz, cz); off += doz;
-        }
-        return true;
+        // selects, not branches: the lanes of a wave cross different axes, and each
+        // branch taken cost as many mask operations as the crossing has arithmetic.
+        // The parameters of the axes not crossed are recomputed to the same values.
+        const bool ax = more && tx == tmn, ay = more && tx != tmn && ty == tmn;
+        const bool az = more && tx != tmn && ty != tmn;
+        px += ax ? gx : 0.f;
+        py += ay ? gy : 0.f;
+        pz += az ? gz : 0.f;
+        tx = tcross(px, rx, cx);
+        ty = tcross(py, ry, cy);
+        tz = tcross(pz, rz, cz);
+        off += ax ? dox : ay ? doy : az ? doz : IdxT(0);
+        return more;
     }
 };
 

@@ -52,9 +52,9 @@ __device__ inline bool col_setup(const ViewRays& vr, const int lo[3], const int 
     const double qx = vr.Q00[0] + (double)ju * vr.U[0];
     const double qy = vr.Q00[1] + (double)ju * vr.U[1];
     const double dx = qx - vr.S[0], dy = qy - vr.S[1];
-    const double l2 = dx * dx + dy * dy;
-    const double il = ray_rsq(l2), l = l2 * il;
-    if (!(l > 0.0)) return false;   // NaN where l2 is 0
+    const double l = sqrt(dx * dx + dy * dy);
+    if (!(l > 0.0)) return false;
+    const double il = 1.0 / l;
     const double u[2] = {dx * il, dy * il};
     const double hc = -(vr.S[0] * u[0] + vr.S[1] * u[1]);
     C.z.hc = hc;
@@ -76,7 +76,7 @@ __device__ inline bool col_setup(const ViewRays& vr, const int lo[3], const int 
             continue;
         }
         const double P0 = floor(oab);
-        const double ru = ray_rcp(u[a]);
+        const double ru = 1.0 / u[a];
         C.P0[a] = (float)P0;
         C.sg[a] = u[a] > 0.0 ? 1 : -1;
         C.r[a] = (float)ru;

@@ -197,8 +197,9 @@ __device__ __forceinline__ bool project_point(const ViewRays& vd, const float X[
 // no view's last round is short; 512 threads on 32 KB of sums put 4 waves on a SIMD
 // where 256 had 2 on volumes of a few hundred bricks.
 // 128^3, 180 views of 192^2: 2.89 ms with 256 threads, views one by one, divisions in the
-// set-up and branches in the walk; 1.70 ms; 1.63 with reciprocals (ray_rcp); 1.42 with
-// selects in the walk (Walker::step).  5 and 6 waves per SIMD spill: 1.74 and 1.79 ms.
+// set-up and branches in the walk, 1.60 ms now.  By steps, forward included: 3.53 -> 2.44
+// (the sequence, 512 threads) -> 2.32 (reciprocals, ray_rcp) -> 2.09 ms (selects in the walk,
+// Walker::step).  At 5 and 6 waves per SIMD it spills: 2.42 and 2.47 ms instead of 2.32.
 template <int kB, typename Tv, typename Tp, typename Tm, typename IdxT>
 __global__ __launch_bounds__(kAdjThreads, 4) void k_backproject_matched(
     RayCfg rc, SinoCfg sc, float scale, uint32_t ssu, uint32_t ssv,

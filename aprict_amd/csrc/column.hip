@@ -90,7 +90,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // First indices s in [0, n) with he[s] > x and with he[s] > y (n if none); he is
 // non-decreasing.  Counted 64 entries at a time: the entries are read at once, where a
 // binary search waits for LDS at every step (64^3 x 90 views of 96^2:
-// 52.0 -> 49.6 us).
+// 2.4 of 52 us).
 __device__ __forceinline__ void first_above(const float* he, int n, float x, float y, int lane, int& sx, int& sy) {
     sx = sy = 0;
     for (int s = 0; s < n; s += 64) {

@@ -59,9 +59,10 @@
 // Precision: P, S and the accumulators are FP64.  The face sums reach h P
 // (about 1e3 rows times 1e3 voxels) over all views, 1e-16 of which is far
 // below the FP32 rounding of the terms.  A ray lying in a z plane (the
-// forward's horizontal rows, |slope| < 1e-20) belongs to the voxel below the
+// forward's horizontal rows, row_flat) belongs to the voxel below the
 // plane, as in the forward; such rays are kept out of P and S and added
-// separately.
+// separately.  (With such a row left in, tau and the row's crossing, both what
+// rounding leaves of 0, would disagree by the row's whole length.)
 #include <algorithm>
 #include <mutex>
 
@@ -194,18 +195,17 @@ __global__ __launch_bounds__(256) void k_gather_prep(RayCfg rc, GCfg gc, const a
     };
     auto scan = [](double v) -> double { return g_scan(v); };
     // yhat of row t, 0 for a row lying in its z plane (the forward's horizontal
-    // row, lane_setup; or a height of exactly 0, by which S could not divide),
-    // whose value goes to yh
+    // row, lane_setup), whose value goes to yh
     double yh = 0.0;
     int ifixh = INT32_MIN;
-    auto yhat = [&](float kv, uint32_t k, double dz, bool flat) -> double {
+    auto yhat = [&](float kv, uint32_t k, bool flat) -> double {
         const double m = fma((double)kv, C.z.dm, C.z.m0);
         const float mf = (float)m;
         const float y = to_f32(sino[(int64_t)p * gc.s0 + (int64_t)j * gc.s1 + (int64_t)k * gc.s2]);
-        if (fabsf(mf) < 1e-20f || dz == 0.0) {
+        if (row_flat(mf)) {
             if (flat) {
                 yh += (double)y;
-                ifixh = (int)ceil(fma(C.z.hc, m, C.z.zc)) - 1;
+                ifixh = (int)ceil(flat_height(C.z.zc)) - 1;
             }
             return 0.0;
         }
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void k_gather_prep(RayCfg rc, GCfg gc, const a
             uint32_t k;
             const double dz = row(t, kv, k);
             fall = !(dz > 0.0);
-            if (hit) yv = yhat(kv, k, dz, true);
+            if (hit) yv = yhat(kv, k, true);
             if (fall && yv != 0.0) sv = -yv * l * g_rcp64(dz);
         }
         // rows of the falling side: 0 .. t0 (t0 included: every falling ray below)
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256) void k_gather_prep(RayCfg rc, GCfg gc, const a
             float kv;
             uint32_t k;
             const double dz = row(t, kv, k);
-            const double yv = hit ? yhat(kv, k, dz, false) : 0.0;
+            const double yv = hit ? yhat(kv, k, false) : 0.0;
             if (yv != 0.0) sv = yv * l * g_rcp64(dz);
         }
         const double is = scan(sv);

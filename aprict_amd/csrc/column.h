@@ -175,18 +175,6 @@ __device__ __forceinline__ int seq_count(const AxisSeq& q, float h, bool strict,
     return k;
 }
 
-// A row whose ray rises by less than 2^-46 per voxel length lies in its z plane: its
-// heights at the source and at the pixel are the same numbers up to the rounding of
-// their differences (1e-16 of the slope's terms), and what that rounding leaves must
-// not say on which side of a grid plane the ray runs.
-__device__ __forceinline__ bool row_flat(float m) { return fabsf(m) < 0x1p-46f; }
-// The height of such a row, zc the source's: a height that rounding alone keeps off a
-// grid plane is the plane's.  A ray in a grid plane belongs to the voxel below it.
-__device__ __forceinline__ double flat_height(double zc) {
-    const double n = rint(zc);
-    return fabs(zc - n) < 0x1p-36 ? n : zc;
-}
-
 // z walk of row kv of a column.  The slope m and the z offset of the
 // row's closest approach, zab, are formed in FP64 (zab carries the crossing
 // positions: an error e in zab moves every crossing by e/m); the plane base

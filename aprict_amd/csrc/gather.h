@@ -14,15 +14,22 @@ struct GView {
     float sx, sy;        // source x, y
     float ax, ay;        // detector point of sub-column 0 minus the source (x, y)
     float bx, by;        // step of the detector point per sub-column (x, y)
-    float orient;        // sign of cross(b, a): cross(b, X - S) * orient > 0 in front
-    int32_t t0;          // rows (z order) whose ray does not rise (dz <= 0); set by the gather pre-pass
     float szlo;          // sz's FP32 rounding residual: the source height is sz + szlo
-    double kb;           // -dz0 / dzs + 1/2 in FP64: tau + 1/2 of the plane through the source
+    int32_t flat;        // the row whose rays lie in their z plane, -1: none
+    float pad;
+    double kb;           // 2 + kappa of the plane through the source: 2 - dz0 / dzs (FP64)
 };
 static_assert(sizeof(GView) == 64, "GView layout");
 
 __device__ __forceinline__ float sub_offset_g(uint32_t s, uint32_t ss) {
     return -0.5f + ((float)s + 0.5f) / (float)ss;
+}
+
+// Height of row t (z order, of NT sub-rows) above the source.
+__device__ __forceinline__ double gather_height(const ViewRays& vr, int flip, uint32_t NT, uint32_t ssv, uint32_t t) {
+    const uint32_t sr = flip ? NT - 1 - t : t;
+    const float kv = (float)(sr / ssv) + sub_offset_g(sr % ssv, ssv);
+    return vr.Q00[2] + (double)kv * vr.V[2] - vr.S[2];
 }
 
 // Whether view p is handled here: upright detector (v parallel to z, u
@@ -36,7 +43,7 @@ __device__ inline bool gather_view(const RayCfg& rc, const ap_proj_spec* __restr
     if (!(s->dspec.v.x == 0.f && s->dspec.v.y == 0.f && s->dspec.v.z != 0.f && s->dspec.u.z == 0.f)) return false;
     const ViewRays vr = make_view_rays(rc, specs, p);
     const double cen[3] = {0.5 * (rc.lo[0] + rc.hi[0]), 0.5 * (rc.lo[1] + rc.hi[1]), 0.5 * (rc.lo[2] + rc.hi[2])};
-    const double Sx = vr.S[0] + cen[0], Sy = vr.S[1] + cen[1], Sz = vr.S[2] + cen[2];
+    const double Sx = vr.S[0] + cen[0], Sy = vr.S[1] + cen[1], Sz = flat_height(vr.S[2] + cen[2]);
     const double c0 = 0.5 / ssu - 0.5;
     const double ax = vr.Q00[0] + c0 * vr.U[0] - vr.S[0], ay = vr.Q00[1] + c0 * vr.U[1] - vr.S[1];
     const double bx = vr.U[0] / ssu, by = vr.U[1] / ssu;
@@ -61,15 +68,23 @@ __device__ inline bool gather_view(const RayCfg& rc, const ap_proj_spec* __restr
     gv.szlo = (float)(Sz - (double)gv.sz);
     gv.dz0 = (float)(vr.Q00[2] + kv_first * vz - vr.S[2]);
     gv.dzs = (float)(fabs(vz) / ssv);
-    gv.kb = 0.5 - (vr.Q00[2] + kv_first * vz - vr.S[2]) / (fabs(vz) / ssv);
+    gv.kb = 2.0 - (vr.Q00[2] + kv_first * vz - vr.S[2]) / (fabs(vz) / ssv);
+    // A flat row's own kappa is that of the source's height: moved up by less than any
+    // crossing resolves (2^-38 rows; FP64 rounding of kappa is 2^-42 at 1000 rows), so that
+    // a plane at that height has the row below it, and no lower plane has.
+    gv.flat = -1;
+    const double tz = rint(gv.kb - 2.0);
+    if (tz >= 0.0 && tz < (double)NT &&
+        row_flat((float)(gather_height(vr, flip, NT, ssv, (uint32_t)tz) / sqrt(ax * ax + ay * ay)))) {
+        gv.flat = (int)tz;
+        gv.kb = tz + 2.0 + 0x1p-38;
+    }
     gv.sx = (float)Sx;
     gv.sy = (float)Sy;
     gv.ax = (float)ax;
     gv.ay = (float)ay;
     gv.bx = (float)bx;
     gv.by = (float)by;
-    gv.orient = (float)orient;
-    gv.t0 = 0;
     return true;
 }
 

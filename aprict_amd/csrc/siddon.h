@@ -65,6 +65,18 @@ __device__ __forceinline__ double ray_rsq(double x) {
     return fma(fma(-h * y, y, 0.5), y, y);
 }
 
+// A row whose ray rises by less than 2^-46 per voxel length lies in its z plane: its
+// heights at the source and at the pixel are the same numbers up to the rounding of
+// their differences (1e-16 of the slope's terms), and what that rounding leaves must
+// not say on which side of a grid plane the ray runs.
+__device__ __forceinline__ bool row_flat(float m) { return fabsf(m) < 0x1p-46f; }
+// The height of such a row, zc the source's: a height that rounding alone keeps off a
+// grid plane is the plane's.  A ray in a grid plane belongs to the voxel below it.
+__device__ __forceinline__ double flat_height(double zc) {
+    const double n = rint(zc);
+    return fabs(zc - n) < 0x1p-36 ? n : zc;
+}
+
 // FP64 -> FP32 per-view constants (CB_project_texture_chunked.cu:308-324 for
 // the pixel centres: centre of pixel (j,k) = pos + (j-(nu-1)/2) u + (k-(nv-1)/2) v).
 __device__ inline ViewRays make_view_rays(const RayCfg& rc, const ap_proj_spec* __restrict__ specs,

@@ -256,13 +256,13 @@ uint64_t ap_backproject_matched_workspace_size(const ap_config_cb_project* cfg,
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): ap_backproject_matched without the workspace argument.
- * The gather's prefix sums go to a 132 MiB scratch array that the library
+ * The gather's prefix sums go to a 64 MiB scratch array that the library
  * holds on each GPU it runs on, from the first call there until the process
  * ends, taken in view chunks that fit it (each chunk adds to vol; results
  * agree with ap_backproject_matched to FP32 rounding).  The call allocates
- * no device memory.  Returns AP_ERR_UNSUPPORTED, with a message, when 8
- * bytes per sub-ray of one view, nu ssu (nv ssv + 40) of them, and the view's
- * records (80 bytes per sub-column) exceed 64 MiB.  All
+ * no device memory.  Returns AP_ERR_UNSUPPORTED, with a message, when one
+ * view of the call needs more than 64 MiB
+ * (ap_backproject_matched_workspace_size(cfg, 1, sino_desc) > 2^26).  All
  * calls on one GPU share its scratch: calls that overlap in time (on other
  * streams or host threads) race.                                           */
 int32_t ap_backproject_matched_noalloc(const ap_config_cb_project* cfg,

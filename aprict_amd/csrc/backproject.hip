@@ -911,8 +911,12 @@ __device__ __forceinline__ void gbc_column(const BpCfg& c, const ViewMap& M, con
     const GbcSoft& g = c.gbc;
     const float r0 = x0 - M.S[0], r1 = x1 - M.S[1];
     const float rxy2 = r0 * r0 + r1 * r1;
-    // hardware square root (about 1 ulp; the IEEE one is a dozen instructions)
-    const float rxy = __builtin_amdgcn_sqrtf(rxy2), il = M.inv_Sxy * __builtin_amdgcn_rsqf(rxy2);
+    // hardware square root (about 1 ulp) and one Newton step: the weight has its cube, and
+    // without the step was up to 10 % further from FP64 than with the IEEE root, whose
+    // dozen instructions cost 3 % of the kernel (the step 0.5 %).  (0 at r_xy = 0)
+    const float iy = __builtin_amdgcn_rsqf(rxy2), il = M.inv_Sxy * iy;
+    const float ry = __builtin_amdgcn_sqrtf(rxy2);
+    const float rxy = __builtin_fmaf(__builtin_fmaf(-ry, ry, rxy2), 0.5f * fminf(iy, AP_BIG), ry);
     const float cr = fminf(1.f, fabsf(r0 * M.S[0] + r1 * M.S[1]) * il);
     const float dr = cr - rxy * g.inv_R;
     const float wh = cr * __builtin_amdgcn_rcpf(fmaxf(1e-9f, cr * cr + dr * dr)) *

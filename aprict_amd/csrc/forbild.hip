@@ -36,8 +36,7 @@ struct Prim {
     int clip_mode[3];
     float rho;
     int cls;
-    float bc[3], br2;   // bounding sphere (centre, squared radius) for culling; br2 NaN: never culled
-    float br;           // its radius
+    float bc[3], br;    // bounding sphere for culling; radius inf or NaN (degenerate shape): never culled
 };
 
 // Radius of a sphere about c holding the primitive: |M^-1 l| <= sigma_max(M^-1) |l|
@@ -64,7 +63,6 @@ __device__ void set_bound(Prim& P, double lr) {
     P.bc[0] = (float)P.c[0];
     P.bc[1] = (float)P.c[1];
     P.bc[2] = (float)P.c[2];
-    P.br2 = (float)(r * r);   // inf or NaN (degenerate shape) never culls
     P.br = (float)r;
 }
 

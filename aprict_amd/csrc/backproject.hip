@@ -594,9 +594,10 @@ __device__ __forceinline__ bool col_inside(const BpCfg& c, const ViewMap& M, con
 // band -- one test per column and view, of the first and last voxel -- a voxel
 // costs the interpolation alone; elsewhere bp_col_views takes the views, with
 // the same sums.  Clamps, range flags, the softening test and 64-bit addresses
-// were two thirds of a voxel's instructions; what is left is bound about
-// equally by the vector units (35 instructions a voxel and view) and the L1's
-// gathers (36 cycles).  FDK at 256^3 from 360 views of 384^2, ramp filter
+// were two thirds of a voxel's instructions; what is left (31 to 33 lane
+// instructions a voxel and view) is bound by L1 accesses where the taps are
+// interpolated (0.92 per CU and cycle; vector issue 0.77), by vector issue where
+// they are nearest pixels (1.17).  FDK at 256^3 from 360 views of 384^2, ramp filter
 // included: 7.8 -> 5.5 ms; nearest pixels at 256^3 from 180 views of 512^2
 // (a SIRT step's backprojection): 6.6 -> 3.1 ms.
 template <int kV, int kZ, typename Tp>
